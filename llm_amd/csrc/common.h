@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <string>
@@ -21,6 +22,20 @@ namespace llmhip {
       return ::llmhip::set_error(LLMHIP_ERR_DEVICE, "llm: %s failed: %s (%s:%d)", #call,         \
                                  hipGetErrorString(e_), __FILE__, __LINE__);                     \
   } while (0)
+
+// Lets kernel K take `bytes` of dynamic LDS on the current device, once per
+// device (the attribute call is slower than a launch).
+template <auto K>
+inline int allow_lds(int bytes) {
+  static std::atomic<uint64_t> done{0};  // a bit per device ordinal
+  int dev = 0;
+  LLM_HIP(hipGetDevice(&dev));
+  const uint64_t bit = 1ull << (dev & 63);
+  if (done.load(std::memory_order_relaxed) & bit) return 0;
+  LLM_HIP(hipFuncSetAttribute((const void*)K, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  done.fetch_or(bit, std::memory_order_relaxed);
+  return 0;
+}
 
 // ggml block geometry (gguf/gguf.go:72-92) for the types with kernels.
 struct QType {

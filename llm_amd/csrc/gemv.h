@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.h"
+#include "resident_plan.h"
 
 namespace llmhip {
 
@@ -123,6 +124,7 @@ struct GemvArgs {
   float *op_dx, *op_bsum;
   int32_t* op_exp;
   uint32_t op_nb;
+  uint32_t up0;  // EPI_GATEUP of the resident product: `up` only of tokens from up0 on
 };
 
 // Bytes of the prepared-activation buffers for ntok tokens of k inputs
@@ -150,6 +152,11 @@ constexpr uint32_t GEMM_MIN_TOKENS = 5;
 // once for the launch, gemm_kernel runs every weight tile over all tokens.
 int prep_launch(const GemvArgs& a, int pro, hipStream_t s);
 int gemm_launch(const GemvArgs& a, uint32_t qtype, int epi, hipStream_t s);
+
+// The product with resident activations (resident.h): prologue (PRO_PLAIN, PRO_RMS) and product in one launch,
+// laid out as res_plan says (p.tt != 0), f32 activations.
+int resident_launch(const GemvArgs& a, const ResArgs& ra, const ResPlan& p, uint32_t qtype, int pro, int epi,
+                    hipStream_t s);
 
 // Bytes of LDS a launch needs, and whether the shape is supported.
 int gemv_launch(const GemvArgs& a, uint32_t qtype, int pro, int epi, hipStream_t s);
@@ -238,6 +245,8 @@ int dequant_launch_qt(const QMat& m, float* out, uint32_t map, uint32_t hd, uint
                       hipStream_t s);
 template <uint32_t QT>
 int gemm_launch_qt(const GemvArgs& a, int epi, hipStream_t s);
+template <uint32_t QT>
+int resident_launch_qt(const GemvArgs& a, const ResArgs& ra, const ResPlan& p, int pro, int epi, hipStream_t s);
 template <uint32_t QT>
 int embed_launch_qt(const QMat& m, const int32_t* tokens, const uint32_t* state, float* x, uint32_t ntok,
                     hipStream_t s);

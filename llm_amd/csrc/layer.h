@@ -50,6 +50,17 @@ uint32_t attn_full_max(uint32_t hd);
 // token, chunks): the merge is left to the output projection's prologue
 // (PRO_MERGE).
 int attn_launch(const AttnArgs& a, uint32_t ntok, hipStream_t s, const AttnOps* ops = nullptr, bool merge = true);
+// The attention of a many-token pass over any number of rows (head size 64), att only: no partials, no merge.
+int attn_flash_launch(const AttnArgs& a, uint32_t ntok, hipStream_t s);
+// The last n rows (from t0) of a wide prefill pass copied to the model's chunk buffers, the non-null ones of x +
+// parts (in order), q with att, and act.  embd and ff multiples of 4.
+struct FinishArgs {
+  const float *x, *parts, *q, *att, *act;
+  float *x_out, *q_out, *att_out, *act_out;
+  uint64_t pstride;
+  uint32_t nparts, t0, n, embd, ff;
+};
+int finish_launch(const FinishArgs& f, hipStream_t s);
 // Greedy sampling from the head's per-workgroup partials, the token written
 // to tokens[step + adv] and out[0], the state advanced by adv; with embd and
 // xn also the sampled token's embedding row into xn (the input of the next

@@ -344,6 +344,314 @@ __global__ __launch_bounds__(HD) void attn_merge_kernel(AttnArgs a, AttnOps ops,
   if (EMIT) emit_operand(ops, t, h * HD + d, o / L);
 }
 
+// Three bf16 parts of f32 values, b0 + b1 + b2 = x to its 24 bits (each part the
+// rounded remainder of the ones before; bf16 has f32's exponent range, so no
+// scaling): f32 products as bf16 matrix products.
+typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+struct Split4 {
+  bf4 p[3];
+};
+__device__ __forceinline__ Split4 split3(f4 x) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  Split4 s;
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    // a pair in one conversion; the parts back to f32 by their bits
+    const uint32_t u0 = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x[0], x[1]}, bf2));
+    const uint32_t u1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x[2], x[3]}, bf2));
+    s.p[i] = __builtin_bit_cast(bf4, (uint64_t)u1 << 32 | u0);
+    if (i < 2) {
+      x[0] -= __uint_as_float(u0 << 16);
+      x[1] -= __uint_as_float(u0 & 0xffff0000u);
+      x[2] -= __uint_as_float(u1 << 16);
+      x[3] -= __uint_as_float(u1 & 0xffff0000u);
+    }
+  }
+  return s;
+}
+__device__ __forceinline__ bf8 join8(const bf4& a, const bf4& b) {
+  return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// D[i][j] += A[i] B[j] for operands in three parts: the six products of parts
+// whose magnitudes reach 2^-24 of the whole, smallest first, each over all
+// (i, j) before the next so that dependent MFMAs are I J apart
+// (v_mfma_f32_16x16x32_bf16: lane l holds A[l % 16][8 (l / 16) ..],
+// B[8 (l / 16) ..][l % 16] and D[4 (l / 16) + i][l % 16]).
+template <int I, int J>
+__device__ __forceinline__ void mfma_split(const bf8 (&a)[I][3], const bf8 (&b)[J][3], f4 (&d)[I][J]) {
+  constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+  for (int k = 0; k < 6; k++)
+#pragma unroll
+    for (int i = 0; i < I; i++)
+#pragma unroll
+      for (int j = 0; j < J; j++) d[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][pa[k]], b[j][pb[k]], d[i][j], 0, 0, 0);
+}
+
+// Causal attention of a many-token pass over any number of cache rows (head
+// size 64): a workgroup of eight waves per (KV head g, group of 64 queries
+// numbered token * GQ + (head - g * GQ) as in attn_mma_kernel), walking the
+// cache in chunks of 32 rows, chunk c by the pair of waves c % 4, 32 queries
+// per wave, the softmax kept running in registers: per query the maximum m,
+// the sum l of e^(s - m) and o = sum e^(s - m) v, rescaled by e^(m_old - m_new)
+// when a chunk raises m (the flash-attention recurrence), the four pairs'
+// sums merged at the end through LDS.  No partials go to memory, and a chunk's
+// rows are read once for 64 queries; the next chunk's are in flight
+// (registers) while the current one goes through the matrix cores.
+// Both products are formed transposed, S^T = K Q^T and O^T = V^T P^T: a lane
+// then holds 8 scores of each of two queries (m, l and the rescaling are its
+// own scalars) and its P values are its own B operand, with the value rows'
+// order in LDS permuted to match, so P never leaves the registers.  f32
+// products by mfma_split on three bf16 parts: 96 MFMAs of 16 cycles per wave
+// and chunk where v_mfma_f32_16x16x4_f32 takes 128 of 32; an operand read
+// from LDS serves both query sets (with 16 queries per wave the LDS reads
+// were the longer chain).
+// Longest walks (the last queries) are started first.
+// Operands in LDS: blocks of 64 16-byte slots per part, operand (row r of 16,
+// k-group j) in slot 4 r + (j ^ (r / 2 % 4)): a wave's reads of a block and the
+// staging's 8-byte writes (a slot's halves) are free of bank conflicts (rows
+// at a padded stride were not: two thirds of the LDS cycles).  Key blocks per
+// 16 rows and 32 dimensions; value blocks (transposed) per 16 dimensions, 64
+// bytes apart so that the four the writes of a wave reach lie in different banks.
+constexpr uint32_t AFL_C = 32;                          // rows of a chunk
+constexpr uint32_t AFL_KB = 3 * 1024, AFL_VB = AFL_KB + 64;  // bytes of a key and of a value block's three parts
+constexpr uint32_t AFL_SPLIT = 4 * AFL_KB + 4 * AFL_VB;      // bytes of one pair's chunk
+__device__ __forceinline__ uint32_t afl_slot(uint32_t row, uint32_t j) { return (4 * row + (j ^ ((row >> 1) & 3))) * 16; }
+
+template <bool KVH>
+__global__ __launch_bounds__(512, 2) void attn_flash_kernel(AttnArgs a, uint32_t ntok) {
+  constexpr uint32_t HD = 64, C = AFL_C;
+  extern __shared__ __align__(16) char fl[];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = wave_id(), grp = lane >> 4, r = lane & 15;
+  const uint32_t pair = wave >> 1, wq = wave & 1, ht = tid & 127;
+  char* Ks = fl + pair * AFL_SPLIT;  // [2 nt][2 st] key blocks, [4 dt] value blocks
+  char* Vt = Ks + 4 * AFL_KB;
+  const uint32_t GQ = a.dgq.d, nq = ntok * GQ;
+  const uint32_t b = gridDim.x - 1 - blockIdx.x, qg = fdiv(b, a.dkv), g = b - qg * a.kv_heads, q0 = qg * 64;
+  const uint32_t pos0 = state_pos(a.state);
+  const uint32_t lim = min(a.rows, pos0 + fdiv(min(q0 + 64, nq) - 1, a.dgq) + 1);  // rows any of its queries sees
+  const uint32_t chunks = (lim + C - 1) / C;
+
+  // the pair's rows of chunk c into registers, dimensions 4 c4 .. of key rows
+  // rg + 8 k and of value rows 4 rg + k; rows at or past lim read the last one
+  // (masked below)
+  const uint32_t rg = ht >> 4, c4 = ht & 15;
+  const uint64_t vbase = (uint64_t)a.ctx * a.kvd + g * HD;
+  f4 kk[4], vv[4];
+  auto load = [&](uint32_t c) {
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      kk[k] = kv_load4<KVH>(a.kv, (uint64_t)min(c * C + rg + 8 * k, lim - 1) * a.kvd + g * HD + 4 * c4);
+      vv[k] = kv_load4<KVH>(a.kv, vbase + (uint64_t)min(c * C + 4 * rg + k, lim - 1) * a.kvd + 4 * c4);
+    }
+  };
+  // ... and from there, split, to LDS: key rows as they are; value rows
+  // transposed, row 16 n + 4 j + e at place 8 j + 4 n + e (the P operand's
+  // order).  Rows past lim become zeros.
+  char* kdst = Ks + (c4 >> 3) * AFL_KB + (c4 & 1) * 8;                 // + slot of (row, c4 / 2 % 4)
+  char* vdst = Vt + (c4 >> 2) * AFL_VB + (rg >> 2) * 8;                // + slot of (dimension % 16, rg % 4)
+  auto store = [&](uint32_t c) {
+    const f4 z = {0, 0, 0, 0};
+    if ((c + 1) * C > lim) {  // uniform
+#pragma unroll
+      for (uint32_t k = 0; k < 4; k++) {
+        if (c * C + rg + 8 * k >= lim) kk[k] = z;
+        if (c * C + 4 * rg + k >= lim) vv[k] = z;
+      }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      const Split4 s = split3(kk[k]);
+      char* d = kdst + (k >> 1) * 2 * AFL_KB + afl_slot(rg + 8 * (k & 1), (c4 >> 1) & 3);
+#pragma unroll
+      for (int i = 0; i < 3; i++) *(bf4*)(d + i * 1024) = s.p[i];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      const Split4 s = split3(f4{vv[0][k], vv[1][k], vv[2][k], vv[3][k]});
+      char* d = vdst + afl_slot(4 * (c4 & 3) + k, rg & 3);
+#pragma unroll
+      for (int i = 0; i < 3; i++) *(bf4*)(d + i * 1024) = s.p[i];
+    }
+  };
+  load(pair);
+
+  // this lane's queries: r of the wave's two sets of 16, their B operands
+  // (dimensions 32 st + 8 grp ..) with the score's scale and log2 e (the
+  // exponentials below are powers of two)
+  uint32_t nd[2];  // causal bounds
+  bf8 Q[2][2][3];  // [st][set][part]
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const uint32_t qa = min(q0 + 32 * wq + 16 * s + r, nq - 1), t = fdiv(qa, a.dgq), h = g * GQ + (qa - t * GQ);
+    nd[s] = pos0 + t + 1;
+    const float qs = a.scale * 1.4426950408889634f;
+    const float* qp = a.q + (uint64_t)t * a.heads * HD + h * HD + 8 * grp;
+#pragma unroll
+    for (int st = 0; st < 2; st++) {
+      const Split4 s0 = split3(*(const f4*)(qp + 32 * st) * qs), s1 = split3(*(const f4*)(qp + 32 * st + 4) * qs);
+#pragma unroll
+      for (int i = 0; i < 3; i++) Q[st][s][i] = join8(s0.p[i], s1.p[i]);
+    }
+  }
+  const uint32_t first = pos0 + fdiv(min(q0 + 32 * wq, nq - 1), a.dgq) + 1;  // the least bound of the wave's queries
+  float M[2] = {-INFINITY, -INFINITY}, L[2] = {0, 0};
+  f4 O[HD / 32][2][2];  // [dt / 2][dt % 2][set]
+#pragma unroll
+  for (uint32_t k = 0; k < HD / 8; k++) O[k / 4][k / 2 % 2][k % 2] = f4{0, 0, 0, 0};
+
+  // Phases: pairs 0 and 1 stage a chunk while pairs 2 and 3, half a step
+  // ahead, compute one (each SIMD has a wave of either), then the other way
+  // round, so that the splitting runs in the shadow of the products.
+  const uint32_t steps = (chunks + 3) / 4, ahead = pair >> 1, slot = afl_slot(r, grp);
+  if (ahead) {
+    store(pair);
+    if (steps > 1) load(pair + 4);
+    __syncthreads();
+  } else {
+    __syncthreads();
+  }
+  for (uint32_t ph = ahead; ph < 2 * steps + ahead; ph++, __syncthreads()) {
+    const uint32_t c = 4 * (ph >> 1) + pair;  // (past the last: every row masked)
+    if (!(ph & 1)) {
+      if (ph >= 2 * steps) continue;
+      store(c);
+      if ((ph >> 1) + 1 < steps) load(c + 4);
+      continue;
+    }
+    f4 S[2][2];  // [nt][set]
+#pragma unroll
+    for (int k = 0; k < 4; k++) S[k / 2][k % 2] = f4{0, 0, 0, 0};
+#pragma unroll
+    for (int st = 0; st < 2; st++) {
+      bf8 K[2][3];
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) K[nt][i] = *(const bf8*)(Ks + (2 * nt + st) * AFL_KB + i * 1024 + slot);
+      mfma_split<2, 2>(K, Q[st], S);
+    }
+    const bool edge = (c + 1) * C > first;  // (uniform) a row past the bound of one of the wave's queries
+    // the lane's 8 scores of a set's query: rows 16 nt + 4 grp + i of the chunk
+    bf8 P[2][3];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const uint32_t lr = c * C + 4 * grp;
+      float m = M[s];
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          if (edge && lr + 16 * nt + i >= nd[s]) S[nt][s][i] = -INFINITY;
+          m = fmaxf(m, S[nt][s][i]);
+        }
+      m = fmaxf(m, xor16(m, lane));
+      m = fmaxf(m, xor32(m, lane));
+      // no row seen yet (m = -inf): nothing to scale, every e of a masked row is 0
+      const float f = m > -INFINITY ? __builtin_amdgcn_exp2f(M[s] - m) : 1.f;
+      float l = 0;
+      f4 e[2];
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          e[nt][i] = __builtin_amdgcn_exp2f(S[nt][s][i] - m);
+          if (edge && lr + 16 * nt + i >= nd[s]) e[nt][i] = 0.f;
+          l += e[nt][i];
+        }
+      const Split4 s0 = split3(e[0]), s1 = split3(e[1]);
+#pragma unroll
+      for (int i = 0; i < 3; i++) P[s][i] = join8(s0.p[i], s1.p[i]);
+      M[s] = m;
+      L[s] = L[s] * f + l;  // the lane's rows; the four lanes of a query are added at the end
+#pragma unroll
+      for (uint32_t k = 0; k < HD / 16; k++) O[k / 2][k % 2][s] *= f;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < HD / 32; k++) {
+      bf8 V[2][3];
+#pragma unroll
+      for (int d = 0; d < 2; d++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) V[d][i] = *(const bf8*)(Vt + (2 * k + d) * AFL_VB + i * 1024 + slot);
+      mfma_split<2, 2>(V, P, O[k]);
+    }
+  }
+  // merge the sums of pairs 1-3 into pair 0's: lane l has query r of each set,
+  // output dimensions 16 dt + 4 grp + i
+  float* mg = (float*)fl + wave * 36 * 64 + lane;  // [set][16 o, m, l][64]
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    L[s] += xor16(L[s], lane);
+    L[s] += xor32(L[s], lane);
+    if (pair) {
+#pragma unroll
+      for (uint32_t k = 0; k < HD / 16; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) mg[(18 * s + 4 * k + i) * 64] = O[k / 2][k % 2][s][i];
+      mg[(18 * s + 16) * 64] = M[s];
+      mg[(18 * s + 17) * 64] = L[s];
+    }
+  }
+  __syncthreads();
+  if (pair) return;
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const uint32_t qd = q0 + 32 * wq + 16 * s + r;
+    if (qd >= nq) continue;
+    // pair 0 holds row 0, which every query sees; a pair that saw none has m = -inf, l = 0
+    float m = M[s];
+#pragma unroll
+    for (int p = 1; p < 4; p++) m = fmaxf(m, mg[(2 * p * 36 + 18 * s + 16) * 64]);
+    float f = __builtin_amdgcn_exp2f(M[s] - m), l = L[s] * f;
+#pragma unroll
+    for (uint32_t k = 0; k < HD / 16; k++) O[k / 2][k % 2][s] *= f;
+#pragma unroll
+    for (int p = 1; p < 4; p++) {
+      const float* o = mg + (2 * p * 36 + 18 * s) * 64;
+      f = __builtin_amdgcn_exp2f(o[16 * 64] - m);
+      l += o[17 * 64] * f;
+#pragma unroll
+      for (uint32_t k = 0; k < HD / 16; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) O[k / 2][k % 2][s][i] += o[(4 * k + i) * 64] * f;
+    }
+    const uint32_t t = fdiv(qd, a.dgq), h = g * GQ + (qd - t * GQ);
+    float* op = a.att + (uint64_t)t * a.heads * HD + h * HD + 4 * grp;
+#pragma unroll
+    for (uint32_t k = 0; k < HD / 16; k++) {
+      f4 o;
+#pragma unroll
+      for (int i = 0; i < 4; i++) o[i] = O[k / 2][k % 2][s][i] / l;
+      *(f4*)(op + 16 * k) = o;
+    }
+  }
+}
+
+int attn_flash_launch(const AttnArgs& a0, uint32_t ntok, hipStream_t s) {
+  if (ntok == 0) return 0;
+  if (a0.hd != 64 || a0.rows == 0 || a0.rows > a0.ctx || a0.kv_heads == 0 || a0.heads % a0.kv_heads)
+    return set_error(LLMHIP_ERR_ARG, "llm: attention: head size %u, %u rows of %u not supported", a0.hd, a0.rows,
+                     a0.ctx);
+  AttnArgs a = a0;
+  a.dgq = fast_div(a.heads / a.kv_heads);
+  a.dkv = fast_div(a.kv_heads);
+  constexpr uint32_t lds = 4 * AFL_SPLIT;
+  static_assert(lds >= 8 * 36 * 64 * 4, "the merge's sums");
+  const uint32_t blocks = (ntok * a.dgq.d + 63) / 64 * a.kv_heads;
+  if (a.kv16) {
+    LLM_TRY(allow_lds<attn_flash_kernel<true>>(lds));
+    hipLaunchKernelGGL(attn_flash_kernel<true>, dim3(blocks), dim3(512), lds, s, a, ntok);
+  } else {
+    LLM_TRY(allow_lds<attn_flash_kernel<false>>(lds));
+    hipLaunchKernelGGL(attn_flash_kernel<false>, dim3(blocks), dim3(512), lds, s, a, ntok);
+  }
+  LLM_HIP(hipGetLastError());
+  return 0;
+}
+
 bool attn_ok(uint32_t hd) { return hd == 64 || hd == 128; }
 
 uint32_t attn_full_max(uint32_t hd) { return hd == 64 ? 256 : 128; }
@@ -596,6 +904,32 @@ __global__ void set_state_kernel(uint32_t* state, uint32_t p) {
 
 int set_state_launch(uint32_t* state, uint32_t p, hipStream_t s) {
   hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, s, state, p);
+  LLM_HIP(hipGetLastError());
+  return 0;
+}
+
+// The last rows of a wide prefill pass where Peek, the head and decode read
+// them: rows [t0, t0 + n) of the given ones of x + its parts, q with att, and
+// act, to rows 0 .. n-1.
+__global__ __launch_bounds__(256) void finish_kernel(FinishArgs f) {
+  const uint64_t t = blockIdx.y, i = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const uint64_t E = f.embd, s = (f.t0 + t) * E + i, d = t * E + i;
+  if (i < E && f.x) {
+    f4 v = *(const f4*)(f.x + s);
+    for (uint32_t p = 0; p < f.nparts; p++) v += *(const f4*)(f.parts + p * f.pstride + s);
+    *(f4*)(f.x_out + d) = v;
+  }
+  if (i < E && f.q) {
+    *(f4*)(f.q_out + d) = *(const f4*)(f.q + s);
+    *(f4*)(f.att_out + d) = *(const f4*)(f.att + s);
+  }
+  if (i < f.ff && f.act) *(f4*)(f.act_out + t * f.ff + i) = *(const f4*)(f.act + (f.t0 + t) * f.ff + i);
+}
+
+int finish_launch(const FinishArgs& f, hipStream_t s) {
+  if (f.n == 0) return 0;
+  const uint32_t cols = f.act ? std::max(f.embd, f.ff) : f.embd;
+  hipLaunchKernelGGL(finish_kernel, dim3((cols / 4 + 255) / 256, f.n), dim3(256), 0, s, f);
   LLM_HIP(hipGetLastError());
   return 0;
 }

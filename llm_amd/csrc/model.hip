@@ -91,6 +91,19 @@ struct Lane {
   void* xprep2 = nullptr;
 };
 
+// The buffers of a wide prefill pass (prefill_wide) of up to cap tokens: the
+// residual stream (two, in turn: each sum of x and its parts goes to the other
+// one); in qp, one after the other, q, the output projection's product and the
+// down projection's parts (at most kp), each dead before the next is written
+// (the parts are what the next RMSNorm adds to x); in act likewise the
+// attention's and the SwiGLU's outputs.
+struct Wide {
+  uint32_t cap = 0, kp = 0;  // cap 0: the model takes the chunked prefill
+  float *x[2] = {nullptr, nullptr}, *qp = nullptr, *act = nullptr;
+};
+constexpr uint32_t WIDE_TOKENS = 1024;  // tokens of a wide pass, at most
+constexpr uint32_t WIDE_KPARTS = 8;     // parts of the down projection, at most
+
 struct Model {
   int device = 0;
   llmhip_limits lim{};
@@ -98,7 +111,7 @@ struct Model {
   uint32_t ctx = 0, pm = 64, smax = 0, kvd = 0;
   uint64_t used = 0;
   std::vector<void*> allocs;
-  uint8_t* arena = nullptr;  // weights, norms, biases, KV caches (allocate)
+  uint8_t* arena = nullptr;  // weights, norms, biases, KV caches, wide prefill buffers (allocate)
   uint64_t arena_cap = 0, arena_used = 0;
   bool sizing = false;
   hipStream_t stream = nullptr;
@@ -152,6 +165,7 @@ struct Model {
   // segment of chunk c in set c % (LANES + 1), and per lane its start and end
   // (prefill_wavefront)
   Lane lanes[LANES];
+  Wide wide;
   int lane = 0;
   std::vector<hipEvent_t> seg_done[LANES + 1];
   hipEvent_t lane_ev[LANES] = {};
@@ -411,15 +425,72 @@ static int allocate_pass(Model& m) {
   return 0;
 }
 
-// The weights, norms, biases and KV caches in one zeroed device arena: one
-// pass sizes it, one hipMalloc and one fill, a second pass carves it (about a
+static ResPlan wide_plan(const QMat& q, uint32_t ntok, int pro, int epi, uint32_t kmax) {
+  return res_plan((uint32_t)q.g.tiles, q.g.nb, ntok, (pro & PRO_RMS) != 0, epi == EPI_QKV, q.g.q.type == LLMHIP_Q4_1,
+                  kmax);
+}
+
+static bool same_types(const Layer& a, const Layer& b) {
+  return a.qkv[0].g.q.type == b.qkv[0].g.q.type && a.o.g.q.type == b.o.g.q.type && a.gu[0].g.q.type == b.gu[0].g.q.type &&
+         a.down.g.q.type == b.down.g.q.type;
+}
+
+// Whether the model's prefill runs as wide passes (its layers' matrices
+// sized): f32 activations, the default chunk (Peek's row numbers are the
+// chunk's), head size 64, one matrix per fused group, and rows that fit a
+// workgroup's LDS; else the chunked prefill.
+static bool wide_fits(const Model& m) {
+  if (m.q8 || m.pm != 64 || m.cfg.head_dim != 64) return false;
+  const Layer* p = nullptr;  // the layer before, whose answer holds for one of the same types
+  for (const Layer& L : m.layers) {
+    if (L.nqkv != 1 || L.ngu != 1) return false;
+    if (!p || !same_types(L, *p))
+      for (uint32_t n : {16u, WIDE_TOKENS})  // (what fits depends on k alone)
+        if (!wide_plan(L.qkv[0], n, PRO_RMS, EPI_QKV, 1).tt || !wide_plan(L.o, n, PRO_PLAIN, EPI_STORE, 1).tt ||
+            !wide_plan(L.gu[0], n, PRO_RMS, EPI_GATEUP, 1).tt ||
+            !wide_plan(L.down, n, PRO_PLAIN, EPI_STORE, WIDE_KPARTS).tt)
+          return false;
+    p = &L;
+  }
+  return true;
+}
+
+// The buffers of wide passes, from the arena (sized or carved like the weights).
+static int wide_buffers(Model& m) {
+  const uint64_t E = m.cfg.embd, F = m.cfg.ff, cap = std::min<uint64_t>(WIDE_TOKENS, (m.ctx + 63) / 64 * 64);
+  Wide& w = m.wide;
+  w.cap = (uint32_t)cap;
+  if (m.sizing) {  // the parts that passes of these lengths take; no pass takes more
+    const Layer* p = nullptr;
+    for (const Layer& L : m.layers) {
+      if (!p || !same_types(L, *p))
+        for (uint32_t n = 64; n <= w.cap; n += 64)
+          w.kp = std::max(w.kp, wide_plan(L.down, n, PRO_PLAIN, EPI_STORE, WIDE_KPARTS).kparts);
+      p = &L;
+    }
+  }
+  LLM_TRY(dalloc_n(m, &w.x[0], cap * E));
+  LLM_TRY(dalloc_n(m, &w.x[1], cap * E));
+  LLM_TRY(dalloc_n(m, &w.act, cap * std::max(E, F)));
+  return dalloc_n(m, &w.qp, w.kp * cap * E);
+}
+
+// The weights, norms, biases, KV caches and (where the model and the budget
+// take them) the wide prefill's buffers in one zeroed device arena: one pass
+// sizes it, one hipMalloc and one fill, a second pass carves it (about a
 // hundred separate allocations cost milliseconds at load and at free).
 static int allocate(Model& m) {
   m.sizing = true;
   m.arena_cap = 0;
   int rc = allocate_pass(m);
+  const uint64_t base = m.arena_cap;
+  if (rc == 0 && wide_fits(m)) rc = wide_buffers(m);
   m.sizing = false;
   if (rc) return rc;
+  if (m.used + m.arena_cap > m.lim.memory_budget) {  // without the wide buffers
+    m.wide = Wide{};
+    m.arena_cap = base;
+  }
   if (m.used + m.arena_cap > m.lim.memory_budget) return over_budget(m);
   LLM_HIP(hipSetDevice(m.device));
   LLM_HIP(hipMalloc((void**)&m.arena, m.arena_cap));
@@ -427,6 +498,7 @@ static int allocate(Model& m) {
   LLM_HIP(hipMemsetAsync(m.arena, 0, m.arena_cap, m.stream));
   m.arena_used = 0;
   LLM_TRY(allocate_pass(m));
+  if (m.wide.cap) LLM_TRY(wide_buffers(m));
   m.allocated = true;
   return 0;
 }
@@ -1078,6 +1150,192 @@ static int prefill_wavefront(Model& m, uint32_t n) {
   return rc;
 }
 
+// The lanes of the chunked prefill (lane 0: the model's own buffers).
+static int lanes_setup(Model& m) {
+  const llmhip_config& c = m.cfg;
+  const uint64_t E = c.embd, F = c.ff, pm = m.pm, H = c.heads;
+  for (int k = 1; k < LANES; k++) {
+    Lane& a = m.lanes[k];
+    if (hipStreamCreateWithFlags(&a.stream, hipStreamNonBlocking) != hipSuccess)
+      return set_error(LLMHIP_ERR_DEVICE, "llm: hipStreamCreate failed");
+    LLM_TRY(dalloc_n(m, &a.x, pm * E));
+    LLM_TRY(dalloc_n(m, &a.q, pm * E));
+    LLM_TRY(dalloc_n(m, &a.att, pm * E));
+    LLM_TRY(dalloc_n(m, &a.act, pm * F));
+    LLM_TRY(dalloc_n(m, &a.gbuf, pm * F));
+    LLM_TRY(dalloc_n(m, &a.pv, pm * H * m.smax * c.head_dim));
+    LLM_TRY(dalloc_n(m, &a.ml, pm * H * m.smax * 2));
+    LLM_TRY(dalloc(m, &a.xprep, xprep_bytes(m.pm, (uint32_t)std::max(c.embd, c.ff))));
+    LLM_TRY(dalloc_n(m, &a.state, 2));
+    LLM_TRY(dalloc(m, &a.xprep2, xprep_bytes(m.pm, (uint32_t)c.ff)));
+  }
+  for (hipEvent_t& e : m.lane_ev)
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+      return set_error(LLMHIP_ERR_DEVICE, "llm: hipEventCreate failed");
+  for (auto& v : m.seg_done) {
+    v.resize((size_t)c.layers + 1);
+    for (hipEvent_t& e : v)
+      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+        return set_error(LLMHIP_ERR_DEVICE, "llm: hipEventCreate failed");
+  }
+  return 0;
+}
+
+// ------------------------------------------------------------ wide prefill
+
+// One wide pass: tokens [a, a + n) of the prompt at positions a .. a + n - 1
+// (the cache holds the rows before), five launches per layer: the RMSNorms are
+// part of the products that need them, and the residual additions part of
+// those RMSNorms (resident.h).  Prompts of more than one chunk take it: the
+// chunked wavefront re-dequantises every weight for every 16 tokens and runs
+// eight launches per layer and 64 tokens (Qwen2.5-0.5B shape on MI355X, us:
+// 65 tokens 1306 -> 1174, 128 1396 -> 1290, 256 2690 -> 1743, 2048 19326 -> 7565);
+// a single chunk stays on it (64 tokens, SmolLM2 shape: 1018 against 1281).
+// The launches go to the stream directly: a prompt length has no graph of its
+// own to build first.
+static int wide_pass(Model& m, uint32_t a, uint32_t n, bool last) {
+  const llmhip_config& c = m.cfg;
+  const Wide& w = m.wide;
+  const uint64_t E = c.embd, F = c.ff, pstride = (uint64_t)w.cap * E;
+  bool head = last;
+  const int nl = pass_layers(m, &head);
+  // the prompt's last chunk, which Peek sees
+  const uint32_t t0 = last ? (a + n - 1) / m.pm * m.pm - a : 0;
+  m.dispatches = 0;
+  m.cur_layer = -1;
+  LLM_TRY(set_state_launch(m.state, a, m.stream));
+  float* x = w.x[0];
+  LLM_TRY(launch_rec(m, "embed", 0, [&]() { return embed_launch(m.embd, m.tokens, m.state, x, n, m.stream); }));
+  ResArgs ra;
+  ResPlan p;
+  // the pass's plans: one per kind of product and weight type (a plan costs more host time than its launch)
+  std::map<std::pair<const char*, uint32_t>, ResPlan> plans;
+  auto go = [&](const char* cls, const GemvArgs& g, const QMat& q, int pro, int epi, uint32_t kmax) -> int {
+    ResPlan& kept = plans[{cls, q.g.q.type}];
+    if (!kept.tt) kept = wide_plan(q, n, pro, epi, kmax);
+    p = kept;
+    ra.rparts = p.rparts;
+    ra.kparts = p.kparts;
+    ra.kunits = p.kunits;
+    ra.ystride = pstride;
+    return launch_rec(m, cls, q.g.gguf_bytes(),
+                      [&]() { return resident_launch(g, ra, p, q.g.q.type, pro, epi, m.stream); });
+  };
+  FinishArgs f{};  // the last chunk's rows, for Peek, the head and decode
+  f.t0 = t0;
+  f.n = n - t0;
+  f.embd = c.embd;
+  f.ff = c.ff;
+  uint32_t nd = 0;  // parts of the latest down projection
+  for (int l = 0; l < nl; l++) {
+    const Layer& L = m.layers[l];
+    m.cur_layer = l;
+    {
+      GemvArgs g = base_args(m, L.qkv[0], n);
+      g.x = x;
+      g.ldx = (uint32_t)E;
+      g.nw = L.attn_norm;
+      g.y = w.qp;
+      g.bias = L.bias;
+      g.cs = m.cs;
+      g.kv = L.kv;
+      g.nq = c.embd;
+      g.nk = m.kvd;
+      g.kvd = m.kvd;
+      g.ctx = m.ctx;
+      g.neox = c.rope_neox;
+      ra = ResArgs{};
+      ra.parts = w.qp;
+      ra.pstride = pstride;
+      ra.nparts = nd;
+      if (nd) ra.xout = x = x == w.x[0] ? w.x[1] : w.x[0];
+      LLM_TRY(go("k1", g, L.qkv[0], PRO_RMS, EPI_QKV, 1));
+    }
+    {
+      AttnArgs t = attn_args(m, L);
+      t.q = w.qp;
+      t.att = w.act;
+      t.rows = std::min(a + n, m.ctx);
+      t.split = 0;
+      // two queries per workgroup while one chunk of rows covers the pass, 64 per workgroup past that (at 256
+      // positions even: 15.6 against 13.6 us at 14 heads, the other way at 9)
+      const bool one = a + n <= attn_full_max(64);
+      LLM_TRY(launch_rec(m, "k2", 2ull * (a + n) * m.kvd * (m.kv16 ? 2 : 4),
+                         [&]() { return one ? attn_launch(t, n, m.stream) : attn_flash_launch(t, n, m.stream); }));
+    }
+    if (last && l + 1 == nl) {  // before the output projection takes q's place
+      f.q = w.qp;
+      f.att = w.act;
+      f.q_out = m.q;
+      f.att_out = m.att;
+      LLM_TRY(launch_rec(m, "finish", 0, [&]() { return finish_launch(f, m.stream); }));
+    }
+    {
+      GemvArgs g = base_args(m, L.o, n);
+      g.x = w.act;
+      g.ldx = (uint32_t)E;
+      g.y = w.qp;
+      g.ldy = (uint32_t)E;
+      ra = ResArgs{};
+      LLM_TRY(go("k3", g, L.o, PRO_PLAIN, EPI_STORE, 1));
+    }
+    {
+      GemvArgs g = base_args(m, L.gu[0], n);
+      g.x = x;
+      g.ldx = (uint32_t)E;
+      g.nw = L.ffn_norm;
+      g.y = w.act;
+      g.ff = c.ff;
+      if (last && l + 1 == nl) {  // Peek("up")
+        g.up = m.gbuf - t0 * F;
+        g.up0 = t0;
+      }
+      ra = ResArgs{};
+      ra.parts = w.qp;
+      ra.pstride = pstride;
+      ra.nparts = 1;
+      ra.xout = x = x == w.x[0] ? w.x[1] : w.x[0];
+      LLM_TRY(go("k4", g, L.gu[0], PRO_RMS, EPI_GATEUP, 1));
+    }
+    {
+      GemvArgs g = base_args(m, L.down, n);
+      g.x = w.act;
+      g.ldx = (uint32_t)F;
+      g.y = w.qp;
+      g.ldy = (uint32_t)E;
+      ra = ResArgs{};
+      LLM_TRY(go("k5", g, L.down, PRO_PLAIN, EPI_STORE, w.kp));
+      nd = p.kparts;
+    }
+  }
+  m.cur_layer = -1;
+  if (last) {
+    f.x = x;
+    f.parts = w.qp;
+    f.pstride = pstride;
+    f.nparts = nd;
+    f.x_out = m.x;
+    f.q = f.att = nullptr;
+    f.act = nl > 0 ? w.act : nullptr;
+    f.act_out = m.act;
+    LLM_TRY(launch_rec(m, "finish", 0, [&]() { return finish_launch(f, m.stream); }));
+  }
+  m.last_row = n - t0 - 1;
+  if (head) LLM_TRY(rec_head(m, m.last_row, n));
+  else LLM_TRY(rec_adv(m, n));
+  m.stats.dispatches += m.dispatches;
+  m.stats.submits++;
+  return 0;
+}
+
+static int prefill_wide(Model& m, uint32_t n) {
+  for (uint32_t a = 0; a < n; a += m.wide.cap) {
+    const uint32_t b = std::min(a + m.wide.cap, n);
+    LLM_TRY(wide_pass(m, a, b - a, b == n));
+  }
+  return 0;
+}
+
 static PassMat pass_mat(const QMat& q) {
   PassMat p;
   p.qs = q.qs;
@@ -1226,31 +1484,7 @@ int llmhip_model_create(int ordinal, const llmhip_limits* lim, const llmhip_conf
       (rc = dalloc_n(*m, &m->ll, pass_words(c, m->kvd, pass_partials(c, m->ctx)))) || (rc = dalloc_n(*m, &m->pctrl, 4)) ||
       (rc = dalloc_n(*m, &m->ptab, (uint64_t)c.layers)))
     return fail(rc);
-  {  // the prefill lanes: lane 0 is the model's own buffers
-    m->lanes[0] = Lane{m->stream, m->x, m->q, m->att, m->act, m->gbuf, m->pv, m->ml, m->xprep, m->state, m->xprep2};
-    for (int k = 1; k < LANES; k++) {
-      Lane& a = m->lanes[k];
-      if (hipStreamCreateWithFlags(&a.stream, hipStreamNonBlocking) != hipSuccess)
-        return fail(set_error(LLMHIP_ERR_DEVICE, "llm: hipStreamCreate failed"));
-      if ((rc = dalloc_n(*m, &a.x, pm * E)) || (rc = dalloc_n(*m, &a.q, pm * E)) ||
-          (rc = dalloc_n(*m, &a.att, pm * E)) || (rc = dalloc_n(*m, &a.act, pm * F)) ||
-          (rc = dalloc_n(*m, &a.gbuf, pm * F)) || (rc = dalloc_n(*m, &a.pv, pm * H * m->smax * c.head_dim)) ||
-          (rc = dalloc_n(*m, &a.ml, pm * H * m->smax * 2)) ||
-          (rc = dalloc(*m, &a.xprep, xprep_bytes(m->pm, (uint32_t)std::max(c.embd, c.ff)))) ||
-          (rc = dalloc_n(*m, &a.state, 2)) ||
-          (rc = dalloc(*m, &a.xprep2, xprep_bytes(m->pm, (uint32_t)c.ff))))
-        return fail(rc);
-    }
-    for (hipEvent_t& e : m->lane_ev)
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-        return fail(set_error(LLMHIP_ERR_DEVICE, "llm: hipEventCreate failed"));
-    for (auto& v : m->seg_done) {
-      v.resize((size_t)c.layers + 1);
-      for (hipEvent_t& e : v)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-          return fail(set_error(LLMHIP_ERR_DEVICE, "llm: hipEventCreate failed"));
-    }
-  }
+  m->lanes[0] = Lane{m->stream, m->x, m->q, m->att, m->act, m->gbuf, m->pv, m->ml, m->xprep, m->state, m->xprep2};
   // RoPE table in double precision, gpu.go:524-534 (and cpu.go:374-375)
   std::vector<float> cs((size_t)m->ctx * c.head_dim);
   const int hp = c.head_dim / 2;
@@ -1415,6 +1649,7 @@ int llmhip_model_finalize(llmhip_model* h) {
   LLM_HIP(hipStreamSynchronize(m.stream));
   stager_free(&m.st);  // the load is over: release its pinned and device staging
   LLM_TRY(pass_setup(m));
+  if (!m.finalized && !m.wide.cap) LLM_TRY(lanes_setup(m));
   m.stats.submits++;
   m.finalized = true;
   return 0;
@@ -1437,7 +1672,9 @@ int llmhip_model_prefill(llmhip_model* h, const int32_t* ids, int n, float* logi
   memcpy(m.host, ids, (size_t)n * 4);
   LLM_HIP(hipMemcpyAsync(m.tokens, m.host, (size_t)n * 4, hipMemcpyHostToDevice, m.stream));
   bool full = m.layers_limit == 0 || m.layers_limit >= m.cfg.layers;
-  if ((uint32_t)n > m.pm && prefill_lanes() > 1) {
+  if (m.wide.cap && (uint32_t)n > m.pm && m.skip.empty()) {
+    LLM_TRY(prefill_wide(m, (uint32_t)n));
+  } else if ((uint32_t)n > m.pm && prefill_lanes() > 1 && m.lanes[1].stream) {
     LLM_TRY(prefill_wavefront(m, (uint32_t)n));
   } else {
     LLM_TRY(set_state_launch(m.state, 0, m.stream));

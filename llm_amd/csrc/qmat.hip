@@ -125,6 +125,19 @@ int gemm_launch(const GemvArgs& a, uint32_t qtype, int epi, hipStream_t s) {
   return set_error(LLMHIP_ERR_TYPE, "llm: ggml type %u has no GPU kernel", qtype);
 }
 
+int resident_launch(const GemvArgs& a, const ResArgs& ra, const ResPlan& p, uint32_t qtype, int pro, int epi,
+                    hipStream_t s) {
+  if (a.ntok == 0) return 0;
+  if (!p.tt || a.k % 4 || a.ldx % 4)
+    return set_error(LLMHIP_ERR_ARG, "llm: resident product: %u tokens of k=%u have no layout", a.ntok, a.k);
+  switch (qtype) {
+    case LLMHIP_Q4_0: return resident_launch_qt<LLMHIP_Q4_0>(a, ra, p, pro, epi, s);
+    case LLMHIP_Q4_1: return resident_launch_qt<LLMHIP_Q4_1>(a, ra, p, pro, epi, s);
+    case LLMHIP_Q8_0: return resident_launch_qt<LLMHIP_Q8_0>(a, ra, p, pro, epi, s);
+  }
+  return set_error(LLMHIP_ERR_TYPE, "llm: ggml type %u has no GPU kernel", qtype);
+}
+
 int qmat_dequant(const QMat& m, float* out, hipStream_t s) {
   switch (m.g.q.type) {
     case LLMHIP_Q4_0:

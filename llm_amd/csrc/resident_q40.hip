@@ -1,0 +1,6 @@
+// The many-token product with resident activations for one weight type.
+#include "resident.h"
+
+namespace llmhip {
+template int resident_launch_qt<LLMHIP_Q4_0>(const GemvArgs&, const ResArgs&, const ResPlan&, int, int, hipStream_t);
+}  // namespace llmhip
