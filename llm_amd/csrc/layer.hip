@@ -915,9 +915,14 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs f) {
   const uint64_t t = blockIdx.y, i = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   const uint64_t E = f.embd, s = (f.t0 + t) * E + i, d = t * E + i;
   if (i < E && f.x) {
-    f4 v = *(const f4*)(f.x + s);
-    for (uint32_t p = 0; p < f.nparts; p++) v += *(const f4*)(f.parts + p * f.pstride + s);
-    *(f4*)(f.x_out + d) = v;
+    const f4 x = *(const f4*)(f.x + s);
+    if (f.nparts) {
+      f4 v = *(const f4*)(f.parts + s);
+      for (uint32_t p = 1; p < f.nparts; p++) v += *(const f4*)(f.parts + p * f.pstride + s);
+      *(f4*)(f.x_out + d) = v + x;
+    } else {
+      *(f4*)(f.x_out + d) = x;
+    }
   }
   if (i < E && f.q) {
     *(f4*)(f.q_out + d) = *(const f4*)(f.q + s);

@@ -7,6 +7,8 @@
 #include "gemv_impl.h"
 #include "resident_plan.h"
 
+#include <type_traits>
+
 namespace llmhip {
 
 // The epilogues of a tile's row for four consecutive tokens (tok .. tok + 3) of
@@ -57,7 +59,7 @@ __device__ __forceinline__ void epi4(const GemvArgs& a, uint32_t tile, int r, bo
     float* p = y + (uint64_t)tok * a.ldy + lr;
 #pragma unroll
     for (uint32_t i = 0; i < 4; i++)
-      if (ok && i < n) p[i * a.ldy] = EPI == EPI_ACC ? e.c[i] + v[i] : v[i];
+      if (ok && i < n) p[(uint64_t)i * a.ldy] = EPI == EPI_ACC ? e.c[i] + v[i] : v[i];
   }
   if (EPI == EPI_QKV) {
     // bias (qwen2), RoPE of the q and k rows' pairs (cpu.go:284-303, 374-385), K and V into the cache
@@ -119,9 +121,11 @@ __device__ __forceinline__ void epi4(const GemvArgs& a, uint32_t tile, int r, bo
 // streams its part of the row tiles past them.
 //
 // Staging: each lane loads its items (block b, k-group kq of one token: 8
-// elements; the four lanes of a block's row share a 128-byte line), adds the
-// parts of the row (ra.nparts partial products the residual x is the sum
-// with; the first row part's workgroups store the sum), and for PRO_RMS
+// elements; the four lanes of a block's row share a 128-byte line), for PRO_RMS
+// adds up the parts of the row (ra.nparts partial products), then the residual x
+// (last, so that its larger magnitude is rounded once: logits of 701 tokens
+// 2.5e-7 -> 2.0e-7 off 64-bit ones; the first row part's workgroups store the
+// sum), and
 // multiplies by the norm weights, the scale 1/rms following after the product
 // as in the decode kernel.  Per token the largest magnitude over the part of
 // k gives the power of two that puts it in [2^14, 2^15); hi = f16(x 2^e),
@@ -135,6 +139,11 @@ __device__ __forceinline__ void epi4(const GemvArgs& a, uint32_t tile, int r, bo
 // is dequantised once for TT token groups.  The steps (block, tile) are
 // software-pipelined: a step's MFMAs with the scaling of the step before and
 // the dequantisation of the step after between them.
+//
+// A tile's block products are summed in chains of two units (eight blocks), the
+// chains in `tot`: one chain over 896 inputs was 1.18e-7 off 64-bit sums where
+// gemm_kernel, whose waves split k, is 0.95e-7 off; so it is 0.94e-7, for 1% of
+// the time (151936x896 for 64 tokens: 50.7 -> 51.4 us).
 //
 // Bound by VALU issue: at TT = 2 a step is 17 VALU instructions (9 dequantise,
 // 8 scale) beside 4 MFMAs, 84 of the 104 busy kcycles of a SIMD in the gate/up
@@ -150,6 +159,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
   // the instruction fetch of code run once counts; [q; k; v] of 128 tokens 12.8 -> 12.0 us); else two copies, one
   // per register set
   constexpr bool ROLL = GT == 1;
+  constexpr bool LATE = GT == 4;  // the residual read in the epilogue: ahead of it, its registers would spill
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int r = lane & 15, q = lane >> 4;
   const uint32_t nb = a.nb, ng = a.ng;
@@ -221,21 +231,23 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
       for (int i = 0; i < NWL; i++) wl[i] = *(const f4*)(a.nw + min((uint32_t)(tid + i * 64 * NW) * 4, nblk * 32 - 4));
     // loads without a condition (a block past the part reads its last one; it
     // takes no part in the maximum, the sum or the operands)
+    // (the sum's terms: the parts, then x)
+    auto term = [&](uint32_t p) { return (PRO & PRO_RMS) && p < ra.nparts ? ra.parts + p * ra.pstride + row : a.x + row; };
     each([&](int h, int i, uint32_t b) {
-      const float* p = a.x + row + 32 * min(b, nblk - 1);
+      const float* p = term(0) + 32 * min(b, nblk - 1);
       v[h][i][0] = *(const f4*)p;
       v[h][i][1] = *(const f4*)(p + 16);
     });
     if (PRO & PRO_RMS) {
       // parts in one round of loads each, or (rows in one batch of items) PU parts in one
       constexpr int PU = NW == 8 ? 4 : 2;
-      uint32_t p = 0;
+      uint32_t p = 1;
       if (!two)
-        for (; p + 1 < ra.nparts; p += PU) {
+        for (; p < ra.nparts; p += PU) {
           f4 y[PU][NI][2];
 #pragma unroll
           for (int k = 0; k < PU; k++) {
-            const float* xp = ra.parts + min(p + k, ra.nparts - 1) * ra.pstride + row;
+            const float* xp = term(min(p + k, ra.nparts));
 #pragma unroll
             for (int i = 0; i < NI; i++) {
               const uint32_t b = min(ws + i * WPT, nblk - 1);
@@ -245,15 +257,15 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
           }
 #pragma unroll
           for (int k = 0; k < PU; k++)
-            if (p + k < ra.nparts)
+            if (p + k <= ra.nparts)
 #pragma unroll
               for (int i = 0; i < NI; i++) {
                 v[0][i][0] += y[k][i][0];
                 v[0][i][1] += y[k][i][1];
               }
         }
-      for (; p < ra.nparts; p++) {
-        const float* xp = ra.parts + p * ra.pstride + row;
+      for (; p <= ra.nparts; p++) {
+        const float* xp = term(p);
         f4 y[2][NI][2];
         each([&](int h, int i, uint32_t b) {
           y[h][i][0] = *(const f4*)(xp + 32 * min(b, nblk - 1));
@@ -365,13 +377,13 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
 
   // ---- the products
   const h8* xl = xs + r * 4 + (q ^ ((r >> 1) & 3));
-  f4 acc[GT][TT], D[TT];
+  f4 acc[GT][TT], tot[GT][TT], D[TT];
   h8 B, Bn;
   float d = 0.f, dn = 0.f, dp = 0.f, m;
 #pragma unroll
   for (int u = 0; u < GT; u++)
 #pragma unroll
-    for (int t = 0; t < TT; t++) acc[u][t] = f4{0, 0, 0, 0};
+    for (int t = 0; t < TT; t++) acc[u][t] = tot[u][t] = f4{0, 0, 0, 0};
 #pragma unroll
   for (int t = 0; t < TT; t++) D[t] = f4{0, 0, 0, 0};
   auto operands = [&](h8 (&A)[TT][2], uint32_t b) {
@@ -383,9 +395,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
   };
   uint32_t cj = 0, cu = 0;  // the unit in the MFMAs
   Epi4In ein[GT][TT];
-  auto process = [&](WUnit (&W)[GT]) {
+  auto process = [&](WUnit (&W)[GT], auto set) {
+    constexpr bool FOLD = !ROLL && decltype(set)::value == 0;  // this unit starts chains of two units' blocks
     const bool last = cu + 1 == units;
-    if ((EPI == EPI_QKV || EPI == EPI_ACC) && last) {
+    if ((EPI == EPI_QKV || (EPI == EPI_ACC && !LATE)) && last) {
       // the epilogue's inputs, under the tile group's last unit
       const uint32_t tile = t0 + (wave + NW * cj) * GT;
 #pragma unroll
@@ -397,19 +410,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
     h8 A[2][TT][2];
     operands(A[0], bu);
     unit_block<QT, false, true>(W[0], 0, B, d, m);
-    if (QT == LLMHIP_Q4_1) {
-      // the unit's sum of m times the block sums: its four blocks as the k of one f32 MFMA
-      float S[TT];
+    float S[TT];
+    if (QT == LLMHIP_Q4_1)
 #pragma unroll
       for (int t = 0; t < TT; t++) S[t] = bs[min(bu + q, nblk - 1) * TT * 16 + t * 16 + r];
-#pragma unroll
-      for (int u = 0; u < GT; u++) {
-        const uint32_t lo = q & 1 ? W[u].sv.y : W[u].sv.x, hi = q & 1 ? W[u].sv.w : W[u].sv.z;
-        const float mm = f16_hw((q & 2 ? hi : lo) >> 16);  // (0 past the tail)
-#pragma unroll
-        for (int t = 0; t < TT; t++) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[t], mm, acc[u][t], 0, 0, 0);
-      }
-    }
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       if (TAIL && (uint32_t)j >= n) break;
@@ -424,7 +428,15 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
 #pragma unroll
         for (int t = 0; t < TT; t++) Dn[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[j & 1][t][1], B, Dn[t], 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < TT; t++) acc[(u + GT - 1) % GT][t] += dp * D[t];
+        for (int t = 0; t < TT; t++) {
+          f4& c = acc[(u + GT - 1) % GT][t];
+          if (FOLD && j == 0) {
+            tot[(u + GT - 1) % GT][t] += c;
+            c = dp * D[t];
+          } else {
+            c += dp * D[t];
+          }
+        }
         if (u + 1 < GT) unit_block<QT, false, true>(W[u + 1], j, Bn, dn, m);
         else if (j < 3) unit_block<QT, false, true>(W[0], j + 1, Bn, dn, m);
 #pragma unroll
@@ -439,8 +451,27 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
         d = dn;
       }
     }
+    if (QT == LLMHIP_Q4_1) {
+      // the unit's sum of m times the block sums, its four blocks as the k of one f32 MFMA; into the chain that the
+      // unit's other products are in, which it largely cancels (into the one before: errors 12% larger)
+#pragma unroll
+      for (int u = 0; u < GT; u++) {
+        const uint32_t lo = q & 1 ? W[u].sv.y : W[u].sv.x, hi = q & 1 ? W[u].sv.w : W[u].sv.z;
+        const float mm = f16_hw((q & 2 ? hi : lo) >> 16);  // (0 past the tail)
+#pragma unroll
+        for (int t = 0; t < TT; t++) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[t], mm, acc[u][t], 0, 0, 0);
+      }
+    }
     if (!ROLL) fetch(W);
     cu++;
+    if (ROLL && !(cu & 1))
+#pragma unroll
+      for (int u = 0; u < GT; u++)
+#pragma unroll
+        for (int t = 0; t < TT; t++) {
+          tot[u][t] += acc[u][t];
+          acc[u][t] = f4{0, 0, 0, 0};
+        }
     if (!last) return;
     // the tile group is complete
 #pragma unroll
@@ -460,16 +491,17 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
         f4 v;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          v[i] = ldexpf(acc[u][t][i], -ex[i]);
+          v[i] = ldexpf(acc[u][t][i] + tot[u][t][i], -ex[i]);
           if (PRO & PRO_RMS) v[i] *= rs[i];
         }
+        if (EPI == EPI_ACC && LATE) epi4_load<EPI>(ein[u][t], a, tile + u, r, tile + u < t1, g0 * 16 + l);
         epi4<EPI>(a, tile + u, r, tile + u < t1, g0 * 16 + l, v, ein[u][t], yo);
       }
     }
 #pragma unroll
     for (int u = 0; u < GT; u++)
 #pragma unroll
-      for (int t = 0; t < TT; t++) acc[u][t] = f4{0, 0, 0, 0};
+      for (int t = 0; t < TT; t++) acc[u][t] = tot[u][t] = f4{0, 0, 0, 0};
     cu = 0;
     cj++;
   };
@@ -479,15 +511,15 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
 #pragma unroll
       for (int u = 0; u < GT; u++) cur[u] = w[0][u];
       fetch(w[0]);
-      process(cur);
+      process(cur, std::integral_constant<int, 0>());
     }
   } else {
     uint32_t i = 0;
     for (; i + 1 < steps_n; i += 2) {
-      process(w[0]);
-      process(w[1]);
+      process(w[0], std::integral_constant<int, 0>());
+      process(w[1], std::integral_constant<int, 1>());
     }
-    if (i < steps_n) process(w[0]);
+    if (i < steps_n) process(w[0], std::integral_constant<int, 0>());
   }
 }
 
@@ -516,10 +548,8 @@ static int resident_form(const GemvArgs& a, const ResArgs& ra, const ResPlan& p,
   if (f == 1116) return resident_tail<QT, PRO, EPI, 1, 1, 16>(a, ra, p, s);
   if (f == 1216) return resident_tail<QT, PRO, EPI, 1, 2, 16>(a, ra, p, s);
   if (f == 2208) return resident_tail<QT, PRO, EPI, 2, 2, 8>(a, ra, p, s);
-  if constexpr (EPI != EPI_QKV) {
-    if (f == 2216) return resident_tail<QT, PRO, EPI, 2, 2, 16>(a, ra, p, s);
+  if constexpr (EPI != EPI_QKV)
     if (f == 2408) return resident_tail<QT, PRO, EPI, 2, 4, 8>(a, ra, p, s);
-  }
   return set_error(LLMHIP_ERR_ARG, "llm: resident product: no form of %u token groups, %u tiles, %u waves", p.tt, p.gt,
                    p.nw);
 }

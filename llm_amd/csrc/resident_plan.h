@@ -22,7 +22,7 @@ struct ResArgs {
   uint32_t rparts;  // workgroups along the rows, part p tiles [p tiles / rparts, (p + 1) tiles / rparts)
   uint32_t kparts, kunits;  // workgroups along k, each kunits units of four blocks; part p's product goes to y + p * ystride
   uint64_t ystride;
-  // PRO_RMS: the row is x + parts[0] + parts[pstride] + ... (nparts of them, added in that order), and xout
+  // PRO_RMS: the row is parts[0] + parts[pstride] + ... + x (nparts of them, added in that order), and xout
   // (null: not) receives it
   const float* parts;
   uint64_t pstride;
@@ -78,7 +78,7 @@ struct ResForm {
   bool qkv;
 };
 constexpr ResForm RES_FORMS[] = {{1, 1, 8, true},  {1, 1, 16, true},  {1, 2, 16, true},
-                                 {2, 2, 8, true},  {2, 2, 16, false}, {2, 4, 8, false}};
+                                 {2, 2, 8, true},  {2, 4, 8, false}};
 
 // The layout of a product of `tiles` row tiles by nb blocks for ntok tokens
 // (rms: PRO_RMS; qkv: EPI_QKV; sums: Q4_1), over at most kmax parts of k: the
