@@ -248,6 +248,8 @@ int gemm_launch_qt(const GemvArgs& a, int epi, hipStream_t s);
 template <uint32_t QT>
 int resident_launch_qt(const GemvArgs& a, const ResArgs& ra, const ResPlan& p, int pro, int epi, hipStream_t s);
 template <uint32_t QT>
+int resident_ready_qt();
+template <uint32_t QT>
 int embed_launch_qt(const QMat& m, const int32_t* tokens, const uint32_t* state, float* x, uint32_t ntok,
                     hipStream_t s);
 

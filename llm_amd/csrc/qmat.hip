@@ -203,7 +203,44 @@ struct llmhip_qmat {
   hipStream_t stream = nullptr;
   void* xprep = nullptr;  // prepared activations of up to 64 tokens (allocated on first use)
   void* scratch = nullptr;  // this device's noalloc scratch array (resolved at create)
+  ResPlan plan[4];  // of products of 1..16, 17..32, 33..48 and 49..64 tokens (tt = 0: the prefill pair)
 };
+
+// The layouts of a matrix's many-token products, which depend on its shape and
+// the number of 16-token groups alone (laid out once: a layout costs as much
+// host time as a launch).  The resident form is one launch without scratch, but
+// every workgroup stages its tokens' whole rows before its first product, 0.08
+// us a block, where the pair's prep does it once: it pays where a workgroup has
+// several tiles or rows are one unit, and loses on short matrices.  MI355X, us,
+// pair -> resident, in graphs: 896x96 5 tokens 5.9 -> 4.5; 896x896 64 6.2 -> 6.5;
+// 1536x576 5 5.7 -> 6.7; 4864x896 16 6.2 -> 6.4, 24 7.2 -> 6.4, 64 8.7 -> 7.4;
+// 4096x1280 24 7.1 -> 7.7; 4096x2048 24 8.3 -> 10.5; 20000x2048 16 12.2 -> 12.1,
+// 24 18.4 -> 17.6, 64 30.3 -> 24.6; 151936x896 5 26.6 -> 21.8, 64 88.9 -> 49.1
+// (its floor, 119 MB, 22).
+static bool resident_pays(const Geom& g, uint32_t groups) {
+  if (g.rows >> 30) return false;  // (the kernel's row indexes are 32-bit)
+  if (g.nb <= 4) return true;
+  if (g.tiles >= 1024) return groups > 1 || g.nb <= 40;
+  return g.tiles >= 256 && g.nb <= 32 && groups > 1;
+}
+
+static int qmat_plan(llmhip_qmat* q) {
+  const Geom& g = q->m.g;
+  bool any = false;
+  for (uint32_t i = 0; i < 4; i++) {
+    if (!resident_pays(g, i + 1)) continue;
+    q->plan[i] = res_plan((uint32_t)g.tiles, g.nb, 16 * (i + 1), false, false, g.q.type == LLMHIP_Q4_1, 1);
+    any = any || q->plan[i].tt;
+  }
+  if (!any) return 0;
+  LLM_HIP(hipSetDevice(q->m.device));
+  switch (g.q.type) {
+    case LLMHIP_Q4_0: return resident_ready_qt<LLMHIP_Q4_0>();
+    case LLMHIP_Q4_1: return resident_ready_qt<LLMHIP_Q4_1>();
+    case LLMHIP_Q8_0: return resident_ready_qt<LLMHIP_Q8_0>();
+  }
+  return 0;
+}
 
 extern "C" {
 
@@ -344,6 +381,7 @@ int llmhip_qmat_create(int ordinal, uint32_t ggml_type, uint64_t rows, uint64_t 
   llmhip_qmat* q = new llmhip_qmat();
   int rc = qmat_alloc(&q->m, ordinal, ggml_type, rows, k);
   if (rc == 0) rc = noalloc_scratch(ordinal, &q->scratch);
+  if (rc == 0) rc = qmat_plan(q);
   if (rc != 0) {
     qmat_release(&q->m);
     delete q;
@@ -391,11 +429,20 @@ static int qmat_gemv_args(llmhip_qmat* q, const float* x, float* y, int n, GemvA
 }
 
 // One product: the decode kernel below GEMM_MIN_TOKENS tokens, else the
-// prefill pair, whose prepared activations go to `xprep` (xprep_bytes(64, k)
-// bytes; nullptr: the matrix's own buffer, allocated on first use).
+// resident form where the matrix has a layout for it, else the prefill pair,
+// whose prepared activations go to `xprep` (xprep_bytes(64, k) bytes; nullptr:
+// the matrix's own buffer, allocated on first use).
 static int qmat_launch(llmhip_qmat* q, GemvArgs& a, int epi, hipStream_t s, int pro = PRO_PLAIN,
                        void* xprep = nullptr) {
   if (a.ntok < GEMM_MIN_TOKENS) return gemv_launch(a, q->m.g.q.type, pro, epi, s);
+  const ResPlan& p = q->plan[(a.ntok - 1) / 16];
+  if (p.tt && !(pro & PRO_Q8)) {
+    ResArgs ra{};
+    ra.rparts = p.rparts;
+    ra.kparts = p.kparts;
+    ra.kunits = p.kunits;
+    return resident_launch(a, ra, p, q->m.g.q.type, pro, epi, s);
+  }
   if (!xprep) {
     if (!q->xprep) LLM_HIP(hipMalloc(&q->xprep, xprep_bytes(64, (uint32_t)q->m.g.k)));
     xprep = q->xprep;

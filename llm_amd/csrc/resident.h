@@ -554,10 +554,34 @@ static int resident_form(const GemvArgs& a, const ResArgs& ra, const ResPlan& p,
                    p.nw);
 }
 
+template <uint32_t QT, int EPI, int TT, int GT, int NW>
+static int resident_allow() {
+  LLM_TRY((allow_lds<resident_kernel<QT, PRO_PLAIN, EPI, TT, GT, true, NW>>(RES_LDS)));
+  return allow_lds<resident_kernel<QT, PRO_PLAIN, EPI, TT, GT, false, NW>>(RES_LDS);
+}
+
+template <uint32_t QT, int EPI>
+static int resident_allow_epi() {
+  LLM_TRY((resident_allow<QT, EPI, 1, 1, 8>()));
+  LLM_TRY((resident_allow<QT, EPI, 1, 1, 16>()));
+  LLM_TRY((resident_allow<QT, EPI, 1, 2, 16>()));
+  LLM_TRY((resident_allow<QT, EPI, 2, 2, 8>()));
+  return resident_allow<QT, EPI, 2, 4, 8>();
+}
+
+// The current device lets every form of the plain products (EPI_STORE, EPI_ACC)
+// have its LDS: a launch after it makes no other runtime call.
+template <uint32_t QT>
+int resident_ready_qt() {
+  LLM_TRY((resident_allow_epi<QT, EPI_STORE>()));
+  return resident_allow_epi<QT, EPI_ACC>();
+}
+
 template <uint32_t QT>
 int resident_launch_qt(const GemvArgs& a, const ResArgs& ra, const ResPlan& p, int pro, int epi, hipStream_t s) {
   switch (pro * 8 + epi) {
     case PRO_PLAIN * 8 + EPI_STORE: return resident_form<QT, PRO_PLAIN, EPI_STORE>(a, ra, p, s);
+    case PRO_PLAIN * 8 + EPI_ACC: return resident_form<QT, PRO_PLAIN, EPI_ACC>(a, ra, p, s);
     case PRO_RMS * 8 + EPI_QKV: return resident_form<QT, PRO_RMS, EPI_QKV>(a, ra, p, s);
     case PRO_RMS * 8 + EPI_GATEUP: return resident_form<QT, PRO_RMS, EPI_GATEUP>(a, ra, p, s);
   }

@@ -3,4 +3,5 @@
 
 namespace llmhip {
 template int resident_launch_qt<LLMHIP_Q4_0>(const GemvArgs&, const ResArgs&, const ResPlan&, int, int, hipStream_t);
+template int resident_ready_qt<LLMHIP_Q4_0>();
 }  // namespace llmhip
