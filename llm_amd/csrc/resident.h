@@ -179,12 +179,17 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
   float* bs = nws + (PRO & PRO_RMS ? 32 * nblk : 0);         // Q4_1: [nblk][TT * 16] block sums
 
   // ---- the tiles of this wave
+  // (GT == 1) kw waves share a tile, wave ks of them the units ks, ks + kw, ..., their sums added in order at the
+  // end: with few tiles a workgroup one wave each ran all of k in a chain of dependent steps, 55 ns a block, and the
+  // others waited (prefill of 128 tokens, Qwen2.5-0.5B shape: 1389 -> 1329 us).  The plan leaves one round of tiles then.
+  const uint32_t lkw = ROLL ? ra.lkw : 0, kw = 1u << lkw, ks = wave & (kw - 1), slot = wave >> lkw;
   const uint32_t ngrp = (t1 - t0 + GT - 1) / GT;
-  const uint32_t mine = ngrp > (uint32_t)wave ? (ngrp - wave + NW - 1) / NW : 0, steps_n = mine * units;
+  const uint32_t mine = ngrp > slot ? (ngrp - slot + (NW >> lkw) - 1) / (NW >> lkw) : 0;
+  const uint32_t steps_n = units > ks ? mine * ((units - ks + kw - 1) >> lkw) : 0;
   WUnit w[2][GT];
-  uint32_t fj = 0, fu = 0;  // the next unit to fetch: tile group fj of the wave's, unit fu of the part
+  uint32_t fj = 0, fu = ks;  // the next unit to fetch: tile group fj of the wave's, unit fu of the part
   auto fetch = [&](WUnit (&W)[GT]) {
-    const uint32_t ft = t0 + (wave + NW * fj) * GT;
+    const uint32_t ft = t0 + (slot + NW * fj) * GT;
 #pragma unroll
     for (int u = 0; u < GT; u++) {
       const uint32_t t = min(ft + u, t1 - 1);
@@ -203,8 +208,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
         W[u].sv = QT == LLMHIP_Q4_1 ? x.sv : uint4{x.sv.x | x.sv.y << 16, x.sv.z, 0, 0};
       }
     }
-    if (++fu == units) {
-      fu = 0;
+    if ((fu += kw) >= units) {
+      fu = ks;
       fj = min(fj + 1, mine - 1);  // past the end: the last group again (not used)
     }
   };
@@ -393,14 +398,37 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
       A[t][1] = xl[(b * TT + t) * 128 + 64];
     }
   };
-  uint32_t cj = 0, cu = 0;  // the unit in the MFMAs
+  uint32_t cj = 0, cu = ks;  // the unit in the MFMAs
   Epi4In ein[GT][TT];
+  auto finish = [&]() __attribute__((always_inline)) {
+    const uint32_t tile = t0 + (slot + NW * cj) * GT;
+    float* yo = a.y + kp * ra.ystride;
+#pragma unroll
+    for (int t = 0; t < TT; t++) {
+      const uint32_t l = t * 16 + 4 * q;
+      typedef int i4 __attribute__((ext_vector_type(4)));
+      const i4 ex = *(const i4*)(tex + l);
+      f4 rs = f4{1, 1, 1, 1};
+      if (PRO & PRO_RMS) rs = *(const f4*)(trs + l);
+#pragma unroll
+      for (int u = 0; u < GT; u++) {
+        f4 v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          v[i] = ldexpf(acc[u][t][i] + tot[u][t][i], -ex[i]);
+          if (PRO & PRO_RMS) v[i] *= rs[i];
+        }
+        if (EPI == EPI_ACC && LATE) epi4_load<EPI>(ein[u][t], a, tile + u, r, tile + u < t1, g0 * 16 + l);
+        epi4<EPI>(a, tile + u, r, tile + u < t1, g0 * 16 + l, v, ein[u][t], yo);
+      }
+    }
+  };
   auto process = [&](WUnit (&W)[GT], auto set) {
     constexpr bool FOLD = !ROLL && decltype(set)::value == 0;  // this unit starts chains of two units' blocks
-    const bool last = cu + 1 == units;
-    if ((EPI == EPI_QKV || (EPI == EPI_ACC && !LATE)) && last) {
+    const bool last = cu + kw >= units;
+    if ((EPI == EPI_QKV || (EPI == EPI_ACC && !LATE)) && last && ks == 0) {
       // the epilogue's inputs, under the tile group's last unit
-      const uint32_t tile = t0 + (wave + NW * cj) * GT;
+      const uint32_t tile = t0 + (slot + NW * cj) * GT;
 #pragma unroll
       for (int u = 0; u < GT; u++)
 #pragma unroll
@@ -463,8 +491,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
       }
     }
     if (!ROLL) fetch(W);
-    cu++;
-    if (ROLL && !(cu & 1))
+    cu += kw;
+    if (ROLL && !((cu >> lkw) & 1))
 #pragma unroll
       for (int u = 0; u < GT; u++)
 #pragma unroll
@@ -477,32 +505,13 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
 #pragma unroll
     for (int t = 0; t < TT; t++) acc[GT - 1][t] += dp * D[t];
     dp = 0.f;
-    const uint32_t tile = t0 + (wave + NW * cj) * GT;
-    float* yo = a.y + kp * ra.ystride;
-#pragma unroll
-    for (int t = 0; t < TT; t++) {
-      const uint32_t l = t * 16 + 4 * q;
-      typedef int i4 __attribute__((ext_vector_type(4)));
-      const i4 ex = *(const i4*)(tex + l);
-      f4 rs = f4{1, 1, 1, 1};
-      if (PRO & PRO_RMS) rs = *(const f4*)(trs + l);
-#pragma unroll
-      for (int u = 0; u < GT; u++) {
-        f4 v;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          v[i] = ldexpf(acc[u][t][i] + tot[u][t][i], -ex[i]);
-          if (PRO & PRO_RMS) v[i] *= rs[i];
-        }
-        if (EPI == EPI_ACC && LATE) epi4_load<EPI>(ein[u][t], a, tile + u, r, tile + u < t1, g0 * 16 + l);
-        epi4<EPI>(a, tile + u, r, tile + u < t1, g0 * 16 + l, v, ein[u][t], yo);
-      }
-    }
+    if (ROLL && kw > 1) return;  // summed over the tile's waves below
+    finish();
 #pragma unroll
     for (int u = 0; u < GT; u++)
 #pragma unroll
       for (int t = 0; t < TT; t++) acc[u][t] = tot[u][t] = f4{0, 0, 0, 0};
-    cu = 0;
+    cu = ks;
     cj++;
   };
   if constexpr (ROLL) {
@@ -512,6 +521,23 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void resident_kernel(GemvArgs a, R
       for (int u = 0; u < GT; u++) cur[u] = w[0][u];
       fetch(w[0]);
       process(cur, std::integral_constant<int, 0>());
+    }
+    if (kw > 1) {  // uniform over the workgroup
+      f4* ps = (f4*)lds;  // [NW][TT][64], in the operands' place (a wave has at least 1 KB of them per token group)
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < TT; t++) {
+        tot[0][t] += acc[0][t];
+        acc[0][t] = f4{0, 0, 0, 0};
+        ps[(wave * TT + t) * 64 + lane] = tot[0][t];
+      }
+      __syncthreads();
+      if (ks == 0 && mine) {
+        for (uint32_t i = 1; i < kw; i++)
+#pragma unroll
+          for (int t = 0; t < TT; t++) tot[0][t] += ps[((wave + i) * TT + t) * 64 + lane];
+        finish();
+      }
     }
   } else {
     uint32_t i = 0;
@@ -529,6 +555,7 @@ static int resident_go(const GemvArgs& a, const ResArgs& ra0, const ResPlan& p, 
   LLM_TRY((allow_lds<resident_kernel<QT, PRO, EPI, TT, GT, TAIL, NW>>(RES_LDS)));
   ResArgs ra = ra0;
   ra.ttiles = (a.ntok + 16 * TT - 1) / (16 * TT);
+  ra.lkw = p.lkw;
   hipLaunchKernelGGL(k, dim3(res_blocks(ra.ttiles, ra.rparts * ra.kparts)), dim3(64 * NW), p.lds, s, a, ra);
   LLM_HIP(hipGetLastError());
   return 0;

@@ -20,6 +20,7 @@ constexpr uint32_t RES_ITEMS = 10;        // staged items per lane, at most
 struct ResArgs {
   uint32_t ttiles;  // token tiles
   uint32_t rparts;  // workgroups along the rows, part p tiles [p tiles / rparts, (p + 1) tiles / rparts)
+  uint32_t lkw;     // log2 of the waves that share a tile (one tile per group only)
   uint32_t kparts, kunits;  // workgroups along k, each kunits units of four blocks; part p's product goes to y + p * ystride
   uint64_t ystride;
   // PRO_RMS: the row is parts[0] + parts[pstride] + ... + x (nparts of them, added in that order), and xout
@@ -47,7 +48,8 @@ inline uint32_t res_blocks(uint32_t ttiles, uint32_t cols) { return (ttiles * co
 struct ResPlan {
   // token groups, tiles per group and waves of a workgroup; row parts, k parts, units per k part; bytes of LDS
   // (tt = 0: the product does not fit)
-  uint32_t tt = 0, gt = 0, nw = 0, rparts = 0, kparts = 0, kunits = 0, lds = 0;
+  // lkw: log2 of the waves that share a tile
+  uint32_t tt = 0, gt = 0, nw = 0, rparts = 0, kparts = 0, kunits = 0, lds = 0, lkw = 0;
 };
 
 // LDS of nblk blocks of tt token groups: the operands, the staging's partial
@@ -100,15 +102,21 @@ inline ResPlan res_plan(uint32_t tiles, uint32_t nb, uint32_t ntok, bool rms, bo
         if (rp < 1 || rp > tiles) return;
         // the kernel's row split and place are 32-bit
         if ((uint64_t)tiles * rp >> 32 || (uint64_t)groups * rp * k >> 28) return;
-        const uint32_t grps = ((tiles + rp - 1) / rp + f.gt - 1) / f.gt, per = (grps + f.nw - 1) / f.nw;
+        const uint32_t grps = ((tiles + rp - 1) / rp + f.gt - 1) / f.gt, rounds = (groups * rp * k + cus - 1) / cus;
+        const uint32_t per = (grps + f.nw - 1) / f.nw;
         const double busy = std::max(1.0, std::min(grps, f.nw) / 4.0);  // waves at work on a SIMD
-        const uint32_t rounds = (groups * rp * k + cus - 1) / cus;
         const double t = rounds * (ResCost::stage(f.tt, nblk, f.nw) +
                                    per * (f.gt * nblk * ResCost::step(f.tt, f.gt, busy) + 0.3)) +
                          (k - 1) * ResCost::part(ntok);
         if (best.tt && t >= least) return;
         least = t;
-        best = ResPlan{f.tt, f.gt, f.nw, rp, k, kunits, lds};
+        best = ResPlan{f.tt, f.gt, f.nw, rp, k, kunits, lds, 0};
+        // waves share a tile where the workgroup has at most one tile per SIMD (each then waits for its own chain of
+        // steps: prefill of 128 tokens 1389 -> 1329 us; with five tiles, 4864x896 for 64 tokens, 7.9 -> 8.1), each
+        // has a unit, and their sums a place in the operands' LDS (of the last part of k too, the shortest)
+        const uint32_t least_blk = nb - (k - 1) * 4 * kunits;
+        if (f.gt == 1 && grps <= 4 && least_blk * 2 >= f.nw)
+          while (best.lkw < 3 && (grps << (best.lkw + 1)) <= f.nw && kunits >= (2u << best.lkw)) best.lkw++;
       };
       for (uint32_t m = 1; m <= 32; m++) {  // m tile groups for every wave
         const uint32_t rp = (tiles + f.nw * f.gt * m - 1) / (f.nw * f.gt * m);

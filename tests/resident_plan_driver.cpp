@@ -10,7 +10,7 @@
 using namespace llmhip;
 
 int main() {
-  unsigned long plans = 0;
+  unsigned long plans = 0, shared = 0;
   for (uint32_t tiles : {1u, 3u, 7u, 36u, 56u, 72u, 608u, 9496u})
     for (uint32_t nb : {1u, 2u, 4u, 6u, 18u, 28u, 38u, 48u, 78u, 152u, 400u})
       for (uint32_t ntok : {1u, 5u, 16u, 17u, 37u, 64u, 65u, 127u, 128u, 257u, 701u, 1023u, 1024u})
@@ -41,6 +41,13 @@ int main() {
           if (nblk * 32 > ((RES_ITEMS * 8 * 32 + 64 * p.nw * 4 - 1) / (64 * p.nw * 4)) * 64 * p.nw * 4) return bad("norm weights");
           if (p.lds != res_lds(nblk, p.tt, rms, sums) || p.lds > RES_LDS) return bad("lds");
           if (p.rparts < 1 || p.rparts > tiles) return bad("row parts");
+          if (p.lkw) {  // waves that share a tile: one round of tiles, a unit each, and room for their sums
+            const uint32_t last = nb - (p.kparts - 1) * 4 * p.kunits;
+            if (p.gt != 1 || (((tiles + p.rparts - 1) / p.rparts) << p.lkw) > p.nw || p.kunits < (1u << p.lkw) ||
+                last * p.tt * 2048 < p.nw * p.tt * 1024)
+              return bad("shared tiles");
+            shared++;
+          }
           uint32_t at = 0;
           for (uint32_t r = 0; r < p.rparts; r++) {
             const uint32_t t0 = r * tiles / p.rparts, t1 = (r + 1) * tiles / p.rparts;
@@ -58,6 +65,10 @@ int main() {
           for (uint8_t s : seen)
             if (s != 1) return bad("not placed");
         }
+  if (!shared) {
+    printf("no plan shares tiles\n");
+    return 1;
+  }
   printf("ok %lu\n", plans);
   return 0;
 }
